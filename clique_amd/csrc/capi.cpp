@@ -282,7 +282,6 @@ cliqg_status cliqg_plan_multiply(cliqg_plan plan, double alpha, const void* d_x,
         auto& p = P(plan);
         require(ldx >= p.N && ldy >= p.N && k >= 0, "bad leading dimension");
         p.multiply(alpha, d_x, ldx, beta, d_y, ldy, k);
-        CQ_HIP(hipStreamSynchronize(p.stream));
     });
 }
 
