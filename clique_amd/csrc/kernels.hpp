@@ -24,7 +24,7 @@ enum GemmTile : int {
     TILE_STREAM = 8,      // 16 rows and all of K per wave
     TILE_STREAM_32 = 9,   // 32 rows, K over four waves
     TILE_STREAM_16 = 10,  // 16 rows, K over eight waves
-    // 128x128 tiles of packed half-precision parts (FP32 updates)
+    // 128x128 tiles of packed half-precision parts (FP32 updates, on request)
     TILE_SPLIT = 11,
 };
 constexpr bool gemm_tile_streams(int variant) {
@@ -350,8 +350,8 @@ template <class T>
 void launch_gemm_stream(const GemmDesc<T>* d_descs, const int* d_tile_start, int ndesc,
                         int ntiles, int variant, int cols, hipStream_t s);
 // FP32 updates on the half-precision matrix cores (TILE_SPLIT; T float or
-// cfloat): operands of `slab` columns (at most SPLIT_SLAB, a multiple of 64)
-// at a time packed into ws (16-byte runs, the rows' exponents after them), then multiplied. pack_start[i] =
+// cfloat): operands of SPLIT_SLAB columns at a time packed into ws (16-byte
+// runs, the rows' exponents after them), then multiplied. pack_start[i] =
 // number of 32-row blocks (whole 128-row tiles) of the operands before
 // descriptor i; runs: 16-byte runs of all operands, sum of split_runs.
 constexpr int SPLIT_SLAB = 1024;
@@ -361,11 +361,11 @@ struct SplitDesc {
     int eA, eB;        // first exponents of their rows
 };
 template <class T>
-int64_t split_runs(int rows, int K, int slab);
+int64_t split_runs(int rows, int K);
 template <class T>
 void launch_gemm_split(const GemmDesc<T>* d_descs, const SplitDesc* d_split,
                        const int* d_tile_start, const int* d_pack_start, int ndesc, int ntiles,
-                       int npack, int maxK, int slab, void* ws, int64_t runs, hipStream_t s);
+                       int npack, int maxK, void* ws, int64_t runs, hipStream_t s);
 constexpr int SPLIT_FLAGS = G_TRANSB | G_CONJB | G_LOWER | G_ACCUM | G_NEG;
 // chunk_start[i] = number of 1024-element chunks before descriptor i
 template <class T>

@@ -256,9 +256,8 @@ cliqg_status cliqg_plan_set_front(cliqg_plan plan, int s, const void* h_L);
  * fixed blockings). Factors d_vals with the given precision and front type
  * while timing every grouped GEMM launch in each tile shape it admits
  * (32x32 with 16- and 64-deep K chunks, 64x64, 128x128 of four waves for real
- * types, 128x128 of eight waves for complex FP32, 128x128 of half-precision
- * parts for FP32 updates; streaming tiles of 128, 32 and 16 rows for solves)
- * and, with solve_rhs > 0, does the same for a solve
+ * types, 128x128 of eight waves for complex FP32; streaming tiles of 128, 32
+ * and 16 rows for solves) and, with solve_rhs > 0, does the same for a solve
  * with solve_rhs right-hand sides; the fastest shape per launch bucket
  * (working type, role, lower masking, log2 of the launch's 64x64 tile count
  * and of its mean K) goes into a table shared by every plan of the process,
@@ -273,11 +272,12 @@ cliqg_status cliqg_plan_autotune(cliqg_plan plan, const void* d_vals, cliqg_prec
 /* The tuning table as text, one line per tuned bucket: bucket, chosen shape
  * (0: 64x64, 4: 128x128, 5: 32x32, 6: 128x128 eight-wave, 7: 32x32 with
  * 64-deep K chunks, 8, 9 and 10: streaming tiles of 128, 32 and 16 rows, 11:
- * products of half-precision parts) and the milliseconds of the 32x32, 64x64,
- * 128x128, eight-wave 128x128, 64-deep 32x32, the three streaming and the
- * split shapes over the bucket's launches (-1 where not built). h_length gets the full
- * length; at most capacity - 1 characters and a terminating zero are
- * copied to h_buf (which may be NULL to query the length). */
+ * products of half-precision parts, admitted by CLIQG_GEMM_TILE=11 only) and
+ * the milliseconds of the 32x32, 64x64, 128x128, eight-wave 128x128, 64-deep
+ * 32x32, the three streaming and the split shapes over the bucket's launches
+ * (-1 where not built). h_length gets the full length; at most capacity - 1
+ * characters and a terminating zero are copied to h_buf (which may be NULL to
+ * query the length). */
 cliqg_status cliqg_autotune_table(char* h_buf, size_t capacity, size_t* h_length);
 
 /* Timing of the last factorization on the plan's stream (HIP events). */
