@@ -304,20 +304,8 @@ __attribute__((amdgpu_waves_per_eu((TM * TN / (WM * WN) >= 2048) ? 2
         if (c + 1 < nk) chunk(c + 1, std::integral_constant<int, 1>{});
     }
 
-    const W* scaleN = reinterpret_cast<const W*>(d.scaleN);
     const bool lower = d.flags & G_LOWER, accum = d.flags & G_ACCUM, neg = d.flags & G_NEG;
     const bool symm = lower && (d.flags & G_SYMM);
-    // a lane's output columns do not depend on r: their pivots and the
-    // pivots' reciprocals are formed once per 16-column block
-    W sN[BN], rN[BN];
-    if (scaleN) {
-#pragma unroll
-        for (int b = 0; b < BN; ++b) {
-            const int gj = col0 + wj * WTN + b * 16 + (lane & 15);
-            sN[b] = gload(scaleN + (gj < d.N ? gj : 0));
-            rN[b] = pivot_inverse(sN[b]);
-        }
-    }
 #pragma unroll
     for (int a = 0; a < BM; ++a)
 #pragma unroll
@@ -334,13 +322,6 @@ __attribute__((amdgpu_waves_per_eu((TM * TN / (WM * WN) >= 2048) ? 2
                                   accS[a][b][r] - accR[a][b][r] - accI[a][b][r]);
                 else
                     v = make_t<T>(accR[a][b][r], CPX ? accI[a][b][r] : R(0));
-                if (scaleN) {
-                    v = cvt<T>(cvt<W>(v) * rN[b]);
-                    // W = L D from the rounded L, exactly as a pivot-scaled
-                    // update would form it, so updates from W stay consistent
-                    // with the stored factor
-                    if (d.C2) gstore(d.C2 + gi + (int64_t)gj * d.ldc, v * cvt<T>(sN[b]));
-                }
                 if (neg) v = -v;
                 T* p = d.C + gi + (int64_t)gj * d.ldc;
                 if (accum) v = gload(p) + v;

@@ -69,19 +69,17 @@ enum GemmFlags : int {
 // range, no output masks)
 constexpr int STREAM_FLAGS = G_TRANSA | G_CONJA | G_ACCUM | G_NEG | G_KLO | G_KHI;
 
-// C(MxN) (+)= +-op(A)(MxK) diag(scaleK) op(B)(KxN) [diag(scaleN)^{-1}], where
-// op(A) is A, A^T, conj(A) or A^H per the flags (scaleK is never conjugated).
+// C(MxN) (+)= +-op(A)(MxK) diag(scaleK) op(B)(KxN), where op(A) is A, A^T,
+// conj(A) or A^H per the flags (scaleK is never conjugated).
 template <class T>
 struct GemmDesc {
     const T* A;
     const T* B;
     T* C;
     const void* scaleK;   // FP64 field-type pivots multiplying op(A)'s column k (or null)
-    const void* scaleN;   // FP64 field-type pivots dividing output column j (or null)
     int64_t lda, ldb, ldc;
     int M, N, K;
     int flags;
-    T* C2 = nullptr;      // with scaleN: optional second output (ld ldc), C * diag(scaleN)
 };
 
 // Dense copy dst(0:rows, 0:cols) := src(0:rows, 0:cols), both column-major.
