@@ -490,13 +490,18 @@ def main():
                    key=lambda n_: prof32[n_]["ms"])
     g = prof32[upd_name]
     achieved = g["flops"] / (g["ms"] * 1e-3) / 1e12
-    kernel_of = {"gemm_update": "k_gemm<cfloat,64,64,3>", "gemm_update_w8": "k_gemm<cfloat,128,128,3,16,2,4>",
-                 "gemm_update_small": "k_gemm<cfloat,32,32,3>", "gemm_update_large": "k_gemm_split<%s>" % ("cfloat" if cplx else "float"),
-                 "gemm_update_k64": "k_gemm<cfloat,32,32,3,64>"}
+    # the large family is the 128x128 tile of real types, or the products of
+    # half-precision parts where the environment asks for them
+    t = "cfloat" if cplx else "float"
+    split = upd_name == "gemm_update_large" and os.environ.get("CLIQG_GEMM_TILE") == "11"
+    kernel_of = {"gemm_update": f"k_gemm<{t},64,64,3>",
+                 "gemm_update_w8": f"k_gemm<{t},128,128,3,16,2,4>",
+                 "gemm_update_small": f"k_gemm<{t},32,32,3>",
+                 "gemm_update_large": f"k_gemm_split<{t}>" if split else f"k_gemm<{t},128,128,3>",
+                 "gemm_update_k64": f"k_gemm<{t},32,32,3,64>"}
     # complex FP32 products issue three real MFMAs per complex block (Gauss)
     # where the flop convention counts four real multiplications; split ones
     # three half-precision MFMAs per real product
-    split = upd_name == "gemm_update_large"
     mfma_share = 3.0 if split else (0.75 if cplx else 1.0)
     peak = PEAK["fp16" if split else "fp32"]
     traffic, traffic_src = measured_traffic(args.config, args.n, upd_name)
