@@ -182,7 +182,8 @@ cliqg_status cliqg_plan_solve_noalloc(cliqg_plan plan, void* d_x, int ldx, int k
 
 /* y := alpha A x + beta y with the factored values, FP64 (replaces
  * cliq::Multiply, numeric/multiply.hpp:27-166, at world size 1). The product
- * is finished on return. */
+ * is finished on return. A plan with a stream of its own wants its device
+ * current. */
 cliqg_status cliqg_plan_multiply(cliqg_plan plan, double alpha, const void* d_x, int ldx,
                                  double beta, void* d_y, int ldy, int k);
 

@@ -42,3 +42,18 @@ def test_product_is_finished_on_return(device, own):
         torch.cuda.synchronize()
         assert np.array_equal(seen.cpu().numpy(), want)
         assert np.array_equal(y.cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="needs two devices")
+def test_product_is_refused_on_another_device(device):
+    """A plan with its own stream runs its products on the default stream of
+    the current device, which has to be the plan's."""
+    ip, ind, v, dims = P.stencil7(9, 8, 7, 7.0, -1.0)
+    sym = cq.NaturalNestedDissection(*dims, ip, ind, cutoff=32)
+    ft = cq.DistSymmFrontTree(sym, ip, ind)
+    ft.factor(torch.tensor(v, device=device))
+    x = torch.ones(ip.size - 1, dtype=torch.float64, device=device)
+    y = torch.zeros_like(x)
+    with torch.cuda.device(1), pytest.raises(Exception, match="device current"):
+        ft.multiply(x, y)
